@@ -839,11 +839,10 @@ static void capture_graph(NbHandle *h, uint32_t flags, int iters) {
   }
 }
 
-static int nb_evaluate_one(void *handle, uint32_t flags, nb_energies *out) {
+// graphs: the evaluation may be a graph replay and may be recorded
+static int nb_evaluate_one(void *handle, uint32_t flags, nb_energies *out, bool graphs = true) {
   NbHandle *h = (NbHandle *)handle;
   if (!h) return NB_ERR_INVALID;
-  const bool record = !(flags & NB_FLAG_NO_RECORD);
-  flags &= ~NB_FLAG_NO_RECORD;
   if (!h->cell_set || !h->positions_set) {
     h->err = "nb_set_cell and nb_set_positions must be called before nb_evaluate";
     return NB_ERR_INVALID;
@@ -886,7 +885,7 @@ static int nb_evaluate_one(void *handle, uint32_t flags, nb_energies *out) {
         (h->md_graph_dt != h->md_dt || h->md_graph_thermo != h->md_thermo || h->md_graph_t0 != h->md_t0 ||
          h->md_graph_tau != h->md_tau))
       drop_graph(h);
-    if (h->graph_on && h->gexec && h->graph_flags == flags && !h->profiling && !h->want_finite) {
+    if (graphs && h->graph_on && h->gexec && h->graph_flags == flags && !h->profiling && !h->want_finite) {
       // replay; a list that needs rebuilding, an overflowed filtered row or a
       // solve that did not stop within the recorded iterations sends the
       // evaluation down the regular path below
@@ -1012,7 +1011,7 @@ static int nb_evaluate_one(void *handle, uint32_t flags, nb_energies *out) {
     // takes the corrections and records them); no spare correction is
     // recorded, since its early-returning launches cost about as much as
     // two PCG iterations on every replay
-    if (record && h->graph_on && !replayed && status == NB_OK && !h->profiling && !h->used_sor && !h->want_finite) {
+    if (graphs && h->graph_on && !replayed && status == NB_OK && !h->profiling && !h->used_sor && !h->want_finite) {
       int first = e.pcg_iters;
       const bool refining = mutual && h->refine && h->prm.precision == NB_PREC_MIXED;
       h->graph_refine_n = 0;
@@ -1045,14 +1044,8 @@ static int nb_evaluate_one(void *handle, uint32_t flags, nb_energies *out) {
 // With electrostatic alchemistry the energy is the sum of the condensed phase
 // (this handle) and the no-ligand and vapor phases (its two child handles),
 // ParticleMeshEwald.java:894-935; gradients, dU/dX/dL and the virial add up.
-int nb_evaluate(void *handle, uint32_t flags, nb_energies *out) {
-  NbHandle *h = (NbHandle *)handle;
-  if (!h) return NB_ERR_INVALID;
-  if (flags & (NB_FLAG_MD_STEP | NB_FLAG_NO_RECORD)) {
-    h->err = "unknown evaluation flag";
-    return NB_ERR_INVALID;
-  }
-  if (!h->elec_lambda) return nb_evaluate_one(h, flags, out);
+static int evaluate_phases(NbHandle *h, uint32_t flags, nb_energies *out, bool graphs) {
+  if (!h->elec_lambda) return nb_evaluate_one(h, flags, out, graphs);
   if (!h->cell_set || !h->positions_set) {
     h->err = "nb_set_cell and nb_set_positions must be called before nb_evaluate";
     return NB_ERR_INVALID;
@@ -1061,7 +1054,7 @@ int nb_evaluate(void *handle, uint32_t flags, nb_energies *out) {
     HIPCHECK(hipSetDevice(h->device));
     set_ost_phases(h);
     nb_energies e;
-    int status = nb_evaluate_one(h, flags, &e);
+    int status = nb_evaluate_one(h, flags, &e, graphs);
     if (status != NB_OK) return status;
     uint32_t cf = flags & (NB_GRAD | NB_VIRIAL | NB_DUDL | NB_FINITE_PCG);
     NbHandle *kids[2] = {h->child_env, h->child_vap};
@@ -1078,7 +1071,7 @@ int nb_evaluate(void *handle, uint32_t flags, nb_energies *out) {
       }
       k->positions_set = true;
       nb_energies ek;
-      int st = nb_evaluate_one(k, cf, &ek);
+      int st = nb_evaluate_one(k, cf, &ek, graphs);
       if (st != NB_OK) {
         h->err = std::string(c ? "vapor phase: " : "no-ligand phase: ") + k->err;
         return st;
@@ -1116,6 +1109,16 @@ int nb_evaluate(void *handle, uint32_t flags, nb_energies *out) {
   } catch (std::exception &ex) {
     return fail(h, ex, NB_ERR_HIP);
   }
+}
+
+int nb_evaluate(void *handle, uint32_t flags, nb_energies *out) {
+  NbHandle *h = (NbHandle *)handle;
+  if (!h) return NB_ERR_INVALID;
+  if (flags & NB_FLAG_MD_STEP) {
+    h->err = "unknown evaluation flag";
+    return NB_ERR_INVALID;
+  }
+  return evaluate_phases(h, flags, out, true);
 }
 
 // Evaluate several independent systems (one handle each) together.  When
@@ -1284,12 +1287,8 @@ void nb_destroy(void *handle) {
 
 }  // extern "C"
 
-// the starting accelerations of nb_md_step: the steps after it have their own
-// recording (drift and kick included), so this evaluation is not recorded
-int nb_evaluate_md_start(NbHandle *h, nb_energies *out) {
-  if (h->elec_lambda) return nb_evaluate(h, NB_GRAD, out);
-  return nb_evaluate_one(h, NB_GRAD | NB_FLAG_NO_RECORD, out);
-}
+// an evaluation of nb_md_step with kernel launches only, also in graph mode
+int nb_evaluate_launched(NbHandle *h, nb_energies *out) { return evaluate_phases(h, NB_GRAD, out, false); }
 
 // one velocity-Verlet step of nb_md_step (h->md_dt set): drift, evaluation
 // and kick, recorded and replayed as one graph in graph mode

@@ -479,7 +479,7 @@ int nb_md_step(void *handle, int nsteps, double dt, nb_md_report *out) {
     h->md_dt = dt;
     if (!h->md_accel) {
       // MolecularDynamics.init: accelerations of the starting coordinates
-      int rc = nb_evaluate_md_start(h, &e);
+      int rc = nb_evaluate_launched(h, &e);
       if (rc != NB_OK) return rc;
       hipLaunchKernelGGL(k_md_kick, dim3(nb), dim3(256), 0, h->stream, n3, dt, 1, (const double *)h->d_md_mass,
                          (const double *)h->d_grad, h->d_md_v, h->d_md_a, h->d_md_part, (const int32_t *)nullptr,
@@ -491,13 +491,13 @@ int nb_md_step(void *handle, int nsteps, double dt, nb_md_report *out) {
     }
     for (int step = 0; step < nsteps; step++) {
       int rc;
-      if (h->graph_on && !h->elec_lambda) {
+      if (NB_RECORD_MD_STEPS && h->graph_on && !h->elec_lambda) {
         // the whole step in one recorded graph (drift, evaluation, kick)
         rc = nb_evaluate_md_step(h, &e);
       } else {
         nb_md_drift(h);
         HIPCHECK(hipGetLastError());
-        rc = nb_evaluate(h, NB_GRAD, &e);
+        rc = nb_evaluate_launched(h, &e);
         if (rc == NB_OK) nb_md_kick(h, false);
       }
       if (rc != NB_OK) return rc;

@@ -311,13 +311,17 @@ void nb_md_free(NbHandle *h);
 // internal evaluation flag: the evaluation is one velocity-Verlet step (drift
 // before, kick and thermostat after, all in the recorded graph)
 constexpr uint32_t NB_FLAG_MD_STEP = 1u << 30;
-// and: do not record this evaluation (the next ones will have other flags)
-constexpr uint32_t NB_FLAG_NO_RECORD = 1u << 29;
+// Whether nb_md_step records its steps into a graph in graph mode.  Off: a
+// process that timed dynamics this way ended in a host segmentation fault, on
+// the HIP 7.0 runtime that a process binds when it imports torch first, and the
+// cause is not known (the library's own calls keep the runtime's rules:
+// tests/test_host_calls.py).  Steps take kernel launches.
+constexpr bool NB_RECORD_MD_STEPS = false;
 constexpr int NB_PRED_BLOCKS = 256;
 void nb_md_drift(NbHandle *h);
 void nb_md_kick(NbHandle *h, bool guarded);
 int nb_evaluate_md_step(NbHandle *h, nb_energies *out);
-int nb_evaluate_md_start(NbHandle *h, nb_energies *out);
+int nb_evaluate_launched(NbHandle *h, nb_energies *out);
 void nb_valence_terms(NbHandle *h);
 void nb_valence_gather(NbHandle *h);
 void nb_valence_free(NbHandle *h);

@@ -2,9 +2,8 @@
 velocity-Verlet integrator (MolecularDynamics.dynamic, MolecularDynamics.java:
 1285-1299; VelocityVerlet.java:66-113) over the device integrator of the HIP
 library (nb_md_*): positions, velocities and accelerations stay in device
-memory, each step's evaluation is the ForceFieldEnergy handle's (a graph
-replay in graph mode), and the SCF predictor carries the induced dipoles from
-step to step (ParticleMeshEwald's scfPredictor, ASPC)."""
+memory, each step's evaluation is the ForceFieldEnergy handle's, and the SCF
+predictor carries the induced dipoles from step to step (ParticleMeshEwald's scfPredictor, ASPC)."""
 from __future__ import annotations
 
 import numpy as np
@@ -20,8 +19,9 @@ class MolecularDynamics:
     with the Berendsen thermostat."""
 
     def __init__(self, ffe, masses, scf_predictor=ffi.NB_PRED_ASPC, graph=True, berendsen=None):
-        """berendsen: (temperature K, tau ps) for the Berendsen thermostat
-        (Berendsen.java:99-101), None for NVE."""
+        """graph: put the handle in graph mode (its own evaluations; steps are
+        kernel launches either way); berendsen: (temperature K, tau ps) for the
+        Berendsen thermostat (Berendsen.java:99-101), None for NVE."""
         self.ffe = ffe
         self.mass = np.ascontiguousarray(masses, np.float64)
         self._h = ffe._handle

@@ -293,14 +293,10 @@ int nb_get_scf_predictor(void *handle, double *coef, double *history, int32_t *s
  * steps of dt ps from the handle's current positions, one evaluation per step,
  * positions and velocities staying in device memory; nb_md_get_state copies
  * them out (either may be NULL).  The first step after nb_md_init evaluates
- * the starting accelerations.  In graph mode (nb_set_graph) a whole step --
- * drift, evaluation, kick, kinetic energy and thermostat -- is recorded as
- * one graph and replayed; the kick kernels run only when the evaluation is
- * valid (no list rebuild pending, no filtered row overflowed, the solve
- * converged within the recorded iterations), and a step whose replay is not
- * valid is finished on the regular path from its drifted positions.  Handles
- * with alchemical electrostatics (the OST environment and vapour handles)
- * step with a graph per evaluation. */
+ * the starting accelerations.  Steps are kernel launches in graph mode
+ * (nb_set_graph) too: recording them into graphs is switched off, after a
+ * process that replayed them ended in a host segmentation fault whose cause is
+ * not known. */
 int nb_md_init(void *handle, const double *mass, const double *v0);
 int nb_md_step(void *handle, int nsteps, double dt, nb_md_report *out);
 int nb_md_get_state(void *handle, double *x, double *v);

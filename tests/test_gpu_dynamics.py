@@ -128,6 +128,34 @@ def test_velocity_verlet_matches_oracle(oracle):
     assert abs(rep["potential"] - pe) <= 1e-8 * abs(pe)
 
 
+RECORDED_STEPS_OFF = pytest.mark.skip(reason="nb_md_step records no steps (NB_RECORD_MD_STEPS): a process that "
+                                      "replayed them ended in a host segmentation fault whose cause is not known")
+
+
+def test_nve_energy_conservation_in_graph_mode():
+    """40 steps of 0.5 fs with the predictor: the total energy stays within
+    0.1 % of the kinetic energy of its start, and a handle in graph mode takes
+    the same steps without recording any."""
+    xyz, box, top, p, terms, mass = ubiquitin(polar_eps=1e-7)
+    v0 = velocities(mass, seed=9)
+    runs = []
+    for graph in (True, False):
+        h = md_handle(top, box, p, terms, graph=graph, predictor=ffi.NB_PRED_ASPC)
+        try:
+            h.set_positions(xyz.reshape(-1))
+            h.md_init(mass, v0.reshape(-1))
+            r0 = h.md_step(0, 0.0005)
+            reps = [h.md_step(10, 0.0005) for _ in range(4)]
+            runs.append((r0, reps, *h.md_state()))
+            assert h.graph_replays() == 0
+        finally:
+            h.close()
+    (r0, reps, x, v), (_, _, sx, sv) = runs
+    assert max(abs(r["total"] - r0["total"]) for r in reps) <= 1e-3 * r0["kinetic"]
+    assert np.abs(x - sx).max() <= 1e-9 and rel(v, sv) <= 1e-9
+
+
+@RECORDED_STEPS_OFF
 def test_nve_energy_conservation_and_graph_replay():
     """40 steps of 0.5 fs with the predictor and graph replays: the total
     energy stays within 0.1 % of the kinetic energy of its start, and the
@@ -379,6 +407,7 @@ def test_ls_predictor_saves_iterations_on_a_smooth_path():
     assert sum(its[ffi.NB_PRED_LS][4:]) < sum(its[ffi.NB_PRED_NONE][4:])
 
 
+@RECORDED_STEPS_OFF
 def test_md_step_graph_with_list_rebuilds():
     """Graph mode records a whole velocity-Verlet step (drift, evaluation,
     kick) as one graph.  With a 0.3 A list buffer ubiquitin rebuilds its

@@ -1,0 +1,73 @@
+"""What the library's host code asks the HIP runtime for, on a runtime without
+a device (host_stub): graphs, streams, events and memory are used within the
+runtime's rules, and dynamics records no graph."""
+import numpy as np
+import pytest
+
+import host_stub
+from forcefieldx_amd import ffi
+from forcefieldx_amd.forcefield import NonbondedParams
+from forcefieldx_amd.systems import water_box
+
+PARAMS = NonbondedParams(vdw_cutoff=9.0, ewald_cutoff=7.0, grid=(24, 24, 24), polar_eps=1e-4)
+FORMS = pytest.mark.parametrize("precision", [ffi.NB_PREC_FP64, ffi.NB_PREC_MIXED], ids=["fp64", "mixed"])
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    return host_stub.build(str(tmp_path_factory.mktemp("host")))
+
+
+@pytest.fixture
+def stub(library, monkeypatch):
+    monkeypatch.setattr(ffi, "_lib", None)
+    s = host_stub.Stub(library)
+    s.set()
+    yield s
+    s.set()
+    assert s.faults() == [] and s.counts()["live"] == 0
+
+
+def handle(precision, grid=PARAMS.grid):
+    xyz, box, top = water_box(216, 18.643, seed=1)
+    h = ffi.Handle(ffi.params_from(PARAMS, grid, precision), top)
+    h.set_cell(box)
+    h.set_positions(xyz)
+    return h, xyz, np.ones(top.n)
+
+
+@FORMS
+def test_recorded_evaluations(stub, precision):
+    """Replays with rejections (a list to rebuild) and budgets that shrink:
+    every capture is joined, no graph is destroyed with a launch outstanding,
+    nothing is left behind."""
+    h, _, _ = handle(precision)
+    h.set_graph(True)
+    stub.reset()
+    for step in range(30):
+        bad = int(step % 9 == 8)
+        stub.set(moved=bad, reject=bad, iterations=4 if step % 5 else 1)
+        h.evaluate(ffi.NB_GRAD)
+    c = stub.counts()
+    assert h.graph_replays() >= 15 and c["instantiated"] == c["captures"] >= 4
+    h.close()
+
+
+@FORMS
+def test_dynamics_records_no_graph(stub, precision):
+    """Runs of a graph-mode handle, each with a new predictor, with list
+    rebuilds between steps: neither a capture nor a graph."""
+    h, xyz, mass = handle(precision)
+    h.set_graph(True)
+    h.evaluate(ffi.NB_GRAD)
+    for run in range(3):
+        h.set_scf_predictor(ffi.NB_PRED_ASPC)
+        h.set_positions(xyz)
+        h.md_init(mass, np.zeros(3 * len(mass)))
+        stub.reset()
+        for step in range(12):
+            stub.set(moved=int(step % 5 == 4))
+            assert h.md_step(2, 0.001)["steps"] == 2
+        c = stub.counts()
+        assert c["captures"] == c["instantiated"] == c["replays"] == c["destroyed"] == 0 and c["launches"] > 0
+    h.close()
