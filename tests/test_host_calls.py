@@ -71,3 +71,11 @@ def test_dynamics_records_no_graph(stub, precision):
         c = stub.counts()
         assert c["captures"] == c["instantiated"] == c["replays"] == c["destroyed"] == 0 and c["launches"] > 0
     h.close()
+
+
+@FORMS
+def test_strain_derivatives_leave_no_memory(stub, precision):
+    """A handle that computed the virial frees the grid it kept for it."""
+    h, _, _ = handle(precision)
+    h.evaluate(ffi.NB_GRAD | ffi.NB_VIRIAL)
+    h.close()
