@@ -496,6 +496,25 @@ __device__ __forceinline__ void brick_points(const T *__restrict__ bbuf, int e3,
   }
 }
 
+// One x line assembled from the brick buffer, for lines too long to be
+// transformed beside their table (lines_x).
+template <typename T, int NP>
+__global__ void __launch_bounds__(256) k_brick_line(CX<T> *__restrict__ grid, Bricks bk, const T *__restrict__ bbuf,
+                                                    const double *__restrict__ ctl) {
+  if (ctl && ctl[0] != 0.0) return;  // recorded solve already stopped
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  BrickX *xt = (BrickX *)smem_raw;
+  __shared__ long lt[4];
+  const int N = bk.K[0], line = blockIdx.x;
+  brick_tables<NP>(bk, line, 1, xt, lt);
+  __syncthreads();
+  for (int x = threadIdx.x; x < N; x += 256) {
+    BrickVals<T, NP> r;
+    brick_load<T, NP>(bbuf, bk.ext * bk.ext * bk.ext, xt[x], lt, r);
+    grid[(size_t)line * N + x] = brick_sum<T, NP>(r);
+  }
+}
+
 // Gather: 8 lanes per atom, lane kz < 5 sums one z plane (25 rows of 5
 // points) into fractional derivatives, then the lanes are combined with
 // shuffles.  FULL: all 20 derivatives t000..t111 plus the Cartesian
@@ -1140,13 +1159,22 @@ static bool plane_t(NbHandle *h, int np, bool inv, CX<T> *g, const CX<T> *twx, c
   return false;
 }
 
-// x lines of any length (assembled from the bricks when np > 0)
+// x lines of any length (assembled from the bricks when np > 0).  In FP64 the
+// line, its twiddles and its table exceed 64 KB of LDS from a length of 1,638
+// on; such lines are assembled by a launch of their own.
 template <typename T>
 static void lines_x(NbHandle *h, int np, CX<T> *g, const CX<T> *tw, T s) {
   const int K0 = h->K[0], K1 = h->K[1], K2 = h->K[2], L = lines_per_block(K0);
   const Bricks bk = bricks_of(h);
   const T *bb = (const T *)h->d_bbuf, *nul = nullptr;
-  const size_t sh = sizeof(CX<T>) * ((size_t)L * K0 + K0) + (np ? sizeof(BrickX) * K0 + sizeof(long) * 4 * L + 8 : 0);
+  const size_t sl = sizeof(CX<T>) * ((size_t)L * K0 + K0), st = sizeof(BrickX) * K0 + sizeof(long) * 4 * L + 8;
+  if (np && sl + st > h->lds_max) {
+    const dim3 lines(K1 * K2);
+    if (np == 1) NB_LAUNCH((k_brick_line<T, 1>), lines, dim3(256), sizeof(BrickX) * K0, g, bk, bb, h->ctl);
+    else NB_LAUNCH((k_brick_line<T, 2>), lines, dim3(256), sizeof(BrickX) * K0, g, bk, bb, h->ctl);
+    np = 0;
+  }
+  const size_t sh = np ? sl + st : sl;
   const dim3 G((K1 * K2 + L - 1) / L), B(256);
 #define NB_LX(P) \
   NB_LAUNCH((k_fft_lines<T, LINE_EPT, 0, false, P>), G, B, sh, g, K0, K1, K2, L, factor(K0), tw, s, nul, bk, bb, h->ctl)

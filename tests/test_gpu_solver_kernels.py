@@ -18,6 +18,9 @@ CASES = {
     # name: (waters, grid)
     "648": (216, (24, 24, 24)),
     "711-runtime-size": (237, (21, 28, 35)),
+    # x lines assembled by a launch of their own (FP64; a point every 0.011 A is
+    # no grid for the mixed form: second differences of FP32 values lose 1e4)
+    "711-longest-lines": (237, (1701, 9, 14)),
     "3003": (1001, (40, 40, 40)),
     "9000-unequal-edges": (3000, (60, 48, 72)),
     "66003-collapsed": (22001, (96, 96, 96)),
@@ -53,7 +56,7 @@ def test_fp64_equals_oracle(oracle, name):
     assert np.linalg.norm(u - uo) <= 1e-8 * np.linalg.norm(uo)
 
 
-@pytest.mark.parametrize("name", list(CASES))
+@pytest.mark.parametrize("name", [c for c in CASES if c != "711-longest-lines"])
 def test_mixed_and_replays(name):
     """The mixed form within the 1e-5 bar of FP64, and graph replays equal to
     the recorded evaluation (the energy sums are atomic: 1e-12)."""

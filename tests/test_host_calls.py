@@ -79,3 +79,16 @@ def test_strain_derivatives_leave_no_memory(stub, precision):
     h, _, _ = handle(precision)
     h.evaluate(ffi.NB_GRAD | ffi.NB_VIRIAL)
     h.close()
+
+
+@FORMS
+@pytest.mark.parametrize("edge", [1620, 1680, 2048])
+def test_lds_of_the_longest_lines(stub, precision, edge):
+    """The longest lines a grid may have: no launch asks for more than the
+    64 KB of LDS that the kernels' layouts are kept to."""
+    for grid in ((edge, 9, 14), (9, edge, 14), (9, 14, edge)):
+        h, _, _ = handle(precision, grid)
+        stub.reset()
+        h.evaluate(ffi.NB_GRAD | ffi.NB_VIRIAL)
+        assert 0 < stub.counts()["lds"] <= 65536
+        h.close()
