@@ -586,27 +586,29 @@ void nb_perm_field(NbHandle *h) {
   }
 }
 
-// field of the dipoles currently held in the packed records (d_dip): the
-// Ewald-screened field over the Ewald rows, or (precond) the bare Coulomb +
-// Thole field over the preconditioner rows
-// How the next field over the Ewald rows treats the radial factors (FP64 form
+// How the next field over the Ewald rows treats the radial factors.  FP64 form
 // only: the FP32 loop waits on the record gathers either way, and reading the
-// factors made it slower, 24.8 -> 23.7 us at 20,736 atoms but 236 -> 347 us at
-// 288,000).  The first field of an evaluation stores them for the solve's
-// others: 45 -> 29 us a launch at 20,736 atoms, 250 -> 159 us at 90,003.  The
-// slots grow with the rows' capacity, outside a recording (a recorded
-// evaluation has the capacities of the regular one before it); without the
-// memory the factors are formed each time.
+// factors gained little where the device is not full and lost where it is (a
+// launch at 20,736 atoms 24.8 -> 23.7 us, at 288,000 236 -> 347 us).  The first
+// field of an evaluation stores them for the solve's others: 45 -> 29 us a
+// launch at 20,736 atoms, 250 -> 159 us at 90,003.  The slots, 16 bytes a row
+// entry, grow with the rows' capacity, outside a recording (a recorded
+// evaluation has the capacities of the regular one before it).  They are an
+// option: a size that does not fit a quarter of the free memory, so that rows
+// and other handles find theirs (a cluster without a cutoff has n^2 entries), is
+// not asked for again, and the factors are formed each time.
 int nb_coef_mode(NbHandle *h) {
   if (h->prm.precision == NB_PREC_MIXED) return NB_DIP_FORM;
   const size_t bytes = sizeof(DipCoef<double>) * (size_t)h->n * h->maxew;
   if (bytes > h->ewcoef_cap) {
-    if (h->capturing) return NB_DIP_FORM;
+    if (h->capturing || bytes == h->ewcoef_refused) return NB_DIP_FORM;
     if (h->d_ewcoef) hipFree(h->d_ewcoef);
     h->d_ewcoef = nullptr;
     h->ewcoef_cap = 0;
-    if (hipMalloc(&h->d_ewcoef, bytes) != hipSuccess) {
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) != hipSuccess || bytes > avail / 4 || hipMalloc(&h->d_ewcoef, bytes) != hipSuccess) {
       h->d_ewcoef = nullptr;
+      h->ewcoef_refused = bytes;
       (void)hipGetLastError();
       return NB_DIP_FORM;
     }
@@ -624,6 +626,9 @@ static void dip_field_t(NbHandle *h, const void *rec, double aw, double *f, doub
             PRE ? h->d_npc : h->d_new, PRE ? h->maxpc : h->maxew, h->cell, aw, (DipCoef<T> *)h->d_ewcoef, f, fp, h->ctl);
 }
 
+// field of the dipoles currently held in the packed records (d_dip): the
+// Ewald-screened field over the Ewald rows, or (precond) the bare Coulomb +
+// Thole field over the preconditioner rows
 void nb_dip_field_real(NbHandle *h, double *f, double *fp, bool precond) {
   bool use_recip = !h->cell.aperiodic && h->prm.ewald_alpha > 0.0;
   double aw = (use_recip && !precond) ? h->prm.ewald_alpha : 0.0;

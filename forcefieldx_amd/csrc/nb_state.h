@@ -105,6 +105,7 @@ struct NbHandle {
   // the rows), held from the first field of an evaluation's solve on
   void *d_ewcoef = nullptr;
   size_t ewcoef_cap = 0;          // bytes
+  size_t ewcoef_refused = 0;      // a size that did not fit
   bool ewcoef_held = false;
   int32_t *d_nnb = nullptr, *d_new = nullptr, *d_npc = nullptr, *d_nsp = nullptr;
   int32_t *d_flags = nullptr;     // [0] overflow nbr, [1] overflow ew, [2] overflow pc, [3] rebuild needed

@@ -87,7 +87,9 @@ typedef struct {
   int32_t polarization;     /* NB_POL_* */
   int32_t do_vdw;
   int32_t do_pme;
-  int32_t precision;        /* NB_PREC_* */
+  int32_t precision;        /* NB_PREC_*; NB_PREC_FP64 also keeps 16 bytes per entry of the Ewald rows
+                             * (n^2 entries without a cutoff), when they fit a quarter of the free
+                             * device memory; without them the results are the same */
   int32_t max_scf_iter;     /* 1000 */
   int32_t device;           /* HIP device ordinal */
   /* alchemical vdW softcore (VanDerWaals.setLambda, VanDerWaals.java:599-653) */

@@ -35,10 +35,12 @@ class Stub:
         from forcefieldx_amd import ffi
         self.ffi, self.L = ffi, ffi.load(lib)
         self.L.stub_set.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int]
+        self.L.stub_free.argtypes = [C.c_long]
         self.L.stub_faults.restype = C.c_char_p
 
-    def set(self, fail_bytes=0, moved=0, reject=0, iterations=1):
+    def set(self, fail_bytes=0, moved=0, reject=0, iterations=1, free_bytes=1 << 38):
         self.L.stub_set(fail_bytes, moved, reject, iterations)
+        self.L.stub_free(free_bytes)
 
     def reset(self):
         self.L.stub_reset_counts()
@@ -47,6 +49,11 @@ class Stub:
         v = (C.c_long * len(COUNTS))()
         self.L.stub_counts(v)
         return dict(zip(COUNTS, v))
+
+    def allocations(self):
+        """Bytes of each allocation made since the last reset."""
+        v = (C.c_long * 4096)()
+        return v[:self.L.stub_allocations(v, C.c_long(4096))]
 
     def faults(self):
         return self.L.stub_faults().decode().splitlines()

@@ -57,6 +57,7 @@ struct Exec {
 };
 
 std::map<char *, size_t> device, pinned;
+std::vector<long> sizes;                    // of the allocations since the last reset
 // (registered by the constructors of the other objects, before this one's)
 std::map<const void *, std::string> &kernels() {
   static auto *m = new std::map<const void *, std::string>();
@@ -70,6 +71,7 @@ Capture *active = nullptr;
 
 // set by the driver
 long fail_bytes = 0;                        // allocations of this many bytes or more fail (0: none do)
+long free_bytes = 1l << 38;                 // free device memory, as hipMemGetInfo tells it
 int moved = 0, reject = 0, iterations = 1;
 
 // counted for the driver
@@ -155,6 +157,7 @@ hipError_t allocate(std::map<char *, size_t> &m, void **p, size_t bytes) {
   }
   *p = calloc(1, bytes ? bytes : 1);
   m[(char *)*p] = bytes;
+  sizes.push_back((long)bytes);
   counts[C_LIVE]++;
   return hipSuccess;
 }
@@ -199,11 +202,17 @@ void stub_set(long fail_at, int mv, int rj, int it) {
   reject = rj;
   iterations = it;
 }
+void stub_free(long bytes) { free_bytes = bytes; }
 void stub_counts(long *out) { memcpy(out, counts, sizeof(counts)); }
 void stub_reset_counts() {
   const long live = counts[C_LIVE];
   memset(counts, 0, sizeof(counts));
   counts[C_LIVE] = live;
+  sizes.clear();
+}
+long stub_allocations(long *out, long most) {
+  for (long i = 0; i < most && i < (long)sizes.size(); i++) out[i] = sizes[i];
+  return (long)sizes.size();
 }
 const char *stub_faults() { return faults.c_str(); }
 
@@ -258,6 +267,12 @@ hipError_t hipGetSymbolAddress(void **p, const void *) {
 }
 
 hipError_t hipMalloc(void **p, size_t bytes) { return allocate(device, p, bytes); }
+hipError_t hipMemGetInfo(size_t *f, size_t *t) {
+  forbidden("hipMemGetInfo");
+  *f = (size_t)free_bytes;
+  *t = (size_t)1 << 38;
+  return hipSuccess;
+}
 hipError_t hipFree(void *p) { return release(device, p); }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return allocate(pinned, p, bytes); }
 hipError_t hipHostFree(void *p) { return release(pinned, p); }

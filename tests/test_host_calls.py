@@ -23,6 +23,7 @@ def stub(library, monkeypatch):
     monkeypatch.setattr(ffi, "_lib", None)
     s = host_stub.Stub(library)
     s.set()
+    s.reset()
     yield s
     s.set()
     assert s.faults() == [] and s.counts()["live"] == 0
@@ -92,3 +93,23 @@ def test_lds_of_the_longest_lines(stub, precision, edge):
         h.evaluate(ffi.NB_GRAD | ffi.NB_VIRIAL)
         assert 0 < stub.counts()["lds"] <= 65536
         h.close()
+
+
+def test_radial_factors_are_an_option(stub):
+    """The FP64 form's stored radial factors (16 bytes a row entry, its largest
+    allocation here) are tried once per row capacity and left out when they
+    fail or would take more than a quarter of the free memory."""
+    h, _, _ = handle(ffi.NB_PREC_FP64)
+    h.evaluate(ffi.NB_GRAD)   # the rows' capacities
+    h.close()
+    size = max(stub.allocations())
+    assert size % (16 * h.n) == 0
+    for kw, tries in ((dict(fail_bytes=size), 1), (dict(free_bytes=4 * size - 1), 0)):
+        h, _, _ = handle(ffi.NB_PREC_FP64)
+        stub.set(**kw)
+        stub.reset()
+        for _ in range(3):
+            h.evaluate(ffi.NB_GRAD)
+        assert stub.counts()["failed"] == tries and max(stub.allocations()) < size
+        h.close()
+        stub.set()
