@@ -103,7 +103,7 @@ template <typename T>
 __host__ __device__ size_t ws_map(char *base, int n, int maxa, int maxb, long ntot, Ws<T> *w) {
   size_t off = 0;
   auto take = [&](size_t bytes) -> char * {
-    char *q = base + off;
+    char *q = w ? base + off : nullptr;   // no workspace yet where only its size is asked for
     off += (bytes + 255) & ~(size_t)255;
     return q;
   };

@@ -11,20 +11,25 @@ COUNTS = ("launches", "captures", "instantiated", "replays", "destroyed", "unuse
 
 
 def build(folder):
-    """Compile the host side of every source and the stub into one library."""
+    """Compile the host side of every source and the stub into one library.
+    Undefined behaviour that the host code meets becomes a fault of the stub."""
     from forcefieldx_amd import build as nb
-    flags = ["-O1", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "--cuda-host-only", "-w", "-I", nb.CSRC]
+    flags = ["-O1", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "--cuda-host-only", "-w", "-I", nb.CSRC,
+             "-Xarch_host", "-fsanitize=undefined", "-Xarch_host", "-fsanitize-minimal-runtime"]
     jobs, objs = [], []
     for src in [os.path.join(nb.CSRC, s) for s in nb.SOURCES] + [os.path.join(HERE, "hip_stub.cpp")]:
         obj = os.path.join(folder, os.path.basename(src) + ".o")
         objs.append(obj)
         jobs.append(subprocess.Popen([nb.HIPCC, *flags, "-x", "hip", "-c", src, "-o", obj]))
     assert all(j.wait() == 0 for j in jobs)
-    # the device code that the host objects would carry
-    names = set(re.findall(r"__hip_fatbin_\w+", subprocess.check_output(["nm", "-u", *objs], text=True)))
+    # the device code that the host objects would carry, and the sanitizer's handlers
+    missing = subprocess.check_output(["nm", "-u", *objs], text=True)
     fat = os.path.join(folder, "fatbin.c")
     with open(fat, "w") as f:
-        f.writelines(f"char {n}[8];\n" for n in sorted(names))
+        f.write("void stub_fault(const char *);\n")
+        f.writelines(f"char {n}[8];\n" for n in sorted(set(re.findall(r"__hip_fatbin_\w+", missing))))
+        f.writelines(f'void {n}(void) {{ stub_fault("{n}"); }}\n'
+                     for n in sorted(set(re.findall(r"__ubsan_handle_\w+", missing))))
     lib = os.path.join(folder, "libamoeba_host.so")
     subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", lib, fat, *objs, "-lstdc++", "-lm", "-Wl,-Bsymbolic"])
     return lib

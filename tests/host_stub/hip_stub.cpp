@@ -202,6 +202,7 @@ void stub_set(long fail_at, int mv, int rj, int it) {
   reject = rj;
   iterations = it;
 }
+void stub_fault(const char *what) { fault(what); }
 void stub_free(long bytes) { free_bytes = bytes; }
 void stub_counts(long *out) { memcpy(out, counts, sizeof(counts)); }
 void stub_reset_counts() {
