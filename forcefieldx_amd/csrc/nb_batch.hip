@@ -1788,8 +1788,9 @@ static size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 // marks in `separate` the handles whose evaluation must be repeated on the
 // regular path (a failed solve, which the regular path hands to SOR, or a
 // list cutoff beyond the checked image range).
+// shape: the kernel shape (kShapes), or -1 for the tuner's.
 bool nb_batch_evaluate(NbHandle **hv, int count, uint32_t flags, nb_energies *out, std::vector<char> &separate,
-                       int &status) {
+                       int &status, int shape) {
   if (count <= 0) return false;
   std::vector<NbHandle *> hs(hv, hv + count);
   if (!batch_qualifies(hs, flags)) return false;
@@ -1807,9 +1808,11 @@ bool nb_batch_evaluate(NbHandle **hv, int count, uint32_t flags, nb_energies *ou
     int grow;
     if (mixed) {
       pool_buffers<float>(pl, hs, order, off, bf);
+      bf.shape = shape;
       grow = run_batch<float>(bf, hs, P, order, off, retry);
     } else {
       pool_buffers<double>(pl, hs, order, off, bf);
+      bf.shape = shape;
       grow = run_batch<double>(bf, hs, P, order, off, retry);
     }
     if (!grow) break;
@@ -1888,4 +1891,22 @@ int nb_batch_last_config(int device, int32_t cfg[4], double *kernel_ms) {
   for (int q = 0; q < 4; q++) cfg[q] = pl->last[q];
   if (kernel_ms) *kernel_ms = pl->last_ms;
   return NB_OK;
+}
+
+// nb_evaluate_batch with the batch kernel's shape given (test entry): -1 past
+// the last shape, NB_ERR_INVALID for handles that do not qualify
+extern "C" int nb_test_batch_shape(void *const *handles, int count, nb_energies *out, int shape) {
+  if (!handles || count <= 0) return NB_ERR_INVALID;
+  if (shape < 0 || shape >= kNumShapes) return -1;
+  std::vector<char> separate;
+  int status = NB_OK;
+  try {
+    if (!nb_batch_evaluate((NbHandle **)handles, count, NB_GRAD, out, separate, status, shape)) return NB_ERR_INVALID;
+  } catch (std::exception &e) {
+    ((NbHandle *)handles[0])->err = e.what();
+    return NB_ERR_HIP;
+  }
+  for (char again : separate)
+    if (again && status == NB_OK) status = NB_ERR_SCF_DIVERGED;
+  return status;
 }

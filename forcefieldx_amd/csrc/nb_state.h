@@ -329,7 +329,7 @@ void nb_valence_free(NbHandle *h);
 void nb_finite_adjoint(NbHandle *h);
 void nb_finite_add(NbHandle *h);
 bool nb_batch_evaluate(NbHandle **hv, int count, uint32_t flags, nb_energies *out, std::vector<char> &separate,
-                       int &status);
+                       int &status, int shape = -1);
 int nb_batch_last_config(int device, int32_t cfg[4], double *kernel_ms);
 int nb_batch_evaluate_static(NbHandle **hv, int count, uint32_t flags, nb_energies *out);
 

@@ -170,6 +170,8 @@ def load(path=LIB_PATH):
     L.nb_valence_struct_size.restype = C.c_int
     L.nb_test_convolution.argtypes = [_dp, _dp, C.c_int, C.c_int, C.c_int, C.c_int]
     L.nb_test_convolution.restype = C.c_int
+    L.nb_test_batch_shape.argtypes = [C.POINTER(vp), C.c_int, C.POINTER(NbEnergies), C.c_int]
+    L.nb_test_batch_shape.restype = C.c_int
     _lib = L
     return L
 
@@ -385,6 +387,16 @@ def evaluate_batch_static(handles, flags=NB_GRAD):
     arr = (C.c_void_p * len(handles))(*[h.h for h in handles])
     outs = (NbEnergies * len(handles))()
     rc = L.nb_evaluate_batch_static(arr, len(handles), flags, outs)
+    return [o.as_dict() for o in outs], rc
+
+
+def test_batch_shape(handles, shape):
+    """evaluate_batch with the batch kernel's shape given (test entry); rc -1
+    past the last shape."""
+    L = load()
+    arr = (C.c_void_p * len(handles))(*[h.h for h in handles])
+    outs = (NbEnergies * len(handles))()
+    rc = L.nb_test_batch_shape(arr, len(handles), outs, shape)
     return [o.as_dict() for o in outs], rc
 
 

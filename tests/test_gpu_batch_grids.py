@@ -27,7 +27,7 @@ def rel(a, b):
     return np.linalg.norm(a - b) / np.linalg.norm(b)
 
 
-def evaluate(systems, precision, params):
+def evaluate(systems, precision, params, shape=None):
     hs = []
     for xyz, box, top, grid in systems:
         h = ffi.Handle(ffi.params_from(params, grid, precision), top)
@@ -35,7 +35,7 @@ def evaluate(systems, precision, params):
         h.set_positions(xyz)
         hs.append(h)
     try:
-        e, rc = ffi.evaluate_batch(hs, ffi.NB_GRAD)
+        e, rc = ffi.evaluate_batch(hs, ffi.NB_GRAD) if shape is None else ffi.test_batch_shape(hs, shape)
         assert rc == ffi.NB_OK and ffi.batch_config()["systems"] == len(systems)
         return e, [h.gradient().reshape(-1, 3) for h in hs], [h.induced()[0] for h in hs]
     finally:
@@ -66,6 +66,48 @@ def test_batch_grids_at_the_buffer_edges(oracle, form):
             scale = max(abs(ed[k][q]) for q in ("perm", "pol", "vdw"))
             assert abs(e[k]["total"] - ed[k]["total"]) <= 1e-5 * scale, grid
             assert rel(g[k], gd[k]) <= 1e-5 and rel(u[k], ud[k]) <= 1e-5, grid
+
+
+SHAPES = [(256, 8), (256, 16), (512, 8), (512, 16), (256, 4)]   # threads, lanes per atom
+# factors 7 and 5, odd edges, a pass of 6 beside 5 and 7 and alone, planes above the buffer
+MIXES = [(14, 30, 21), (42, 28, 35), (36, 50, 9), (24, 18, 48), (60, 42, 10), (64, 63, 49), (45, 15, 27), (6 * 7, 6 * 5, 54)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", range(len(SHAPES)), ids=["x".join(map(str, s)) for s in SHAPES])
+def test_every_shape_on_mixed_radices(oracle, shape):
+    """Each shape of the batch kernel by itself, FP64 against the oracle and the
+    mixed form against FP64, so that none depends on what the tuner picks."""
+    systems = [(x, b, t, MIXES[k]) for k, (x, b, t, _) in enumerate(crystal_batch(len(MIXES), seed=11))]
+    print("batch shape", SHAPES[shape], flush=True)
+    e, g, u = evaluate(systems, ffi.NB_PREC_FP64, PARAMS, shape)
+    cfg = ffi.batch_config()
+    assert (cfg["threads"], cfg["lanes"]) == SHAPES[shape]
+    for k, (xyz, box, top, grid) in enumerate(systems):
+        eo, go, uo, _ = oracle.evaluate(oracle.System(xyz, box, top), dataclasses.replace(PARAMS, grid=grid))
+        scale = max(abs(eo[q]) for q in ("perm", "pol", "vdw"))
+        for q in ("perm_recip", "perm_real", "pol", "vdw", "total"):
+            assert abs(e[k][q] - eo[q]) <= 1e-8 * scale, (grid, q, e[k][q], eo[q])
+        assert rel(g[k], go) <= 1e-8 and rel(u[k], uo) <= 1e-8, grid
+        assert e[k]["pcg_iters"] == eo["pcg_iters"], grid
+    p = dataclasses.replace(PARAMS, polar_eps=1e-6)
+    e, g, u = evaluate(systems, ffi.NB_PREC_MIXED, p, shape)
+    ed, gd, ud = evaluate(systems, ffi.NB_PREC_FP64, p, shape)
+    for k, (_, _, _, grid) in enumerate(systems):
+        scale = max(abs(ed[k][q]) for q in ("perm", "pol", "vdw"))
+        for q in ("perm", "pol", "vdw", "total"):
+            assert abs(e[k][q] - ed[k][q]) <= 1e-5 * scale, (grid, q)
+        assert rel(g[k], gd[k]) <= 1e-5 and rel(u[k], ud[k]) <= 1e-5, grid
+
+
+@pytest.mark.gpu
+def test_shape_past_the_last():
+    (xyz, box, top, grid), = crystal_batch(1, seed=11)
+    h = ffi.Handle(ffi.params_from(PARAMS, grid, ffi.NB_PREC_FP64), top)
+    h.set_cell(box)
+    h.set_positions(xyz)
+    assert ffi.test_batch_shape([h], len(SHAPES))[1] == -1 and ffi.test_batch_shape([h], -1)[1] == -1
+    h.close()
 
 
 def test_slab_transforms_stay_in_the_buffer():
