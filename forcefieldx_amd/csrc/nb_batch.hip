@@ -160,6 +160,18 @@ template <typename T> struct FftCap { static constexpr int value = 28672 / sizeo
 // lines (mI their magic number) for each outer one, `lines` in all.
 struct Lines { int I, so, se, lines; uint32_t mI; };
 
+// Butterfly b of a pass of radix R over lines of R nb elements, Ns the transforms'
+// length before it: line (i, o), elements j + k nb read, (jq Ns R + jm) + k Ns
+// written, twiddle of element k at jm k (nb / Ns).
+struct Butterfly { int i, o, j, jq, jm; };
+__host__ __device__ __forceinline__ Butterfly butterfly(int b, int nb, const Lines &ln, int Ns, uint32_t mnb,
+                                                        uint32_t mns) {
+  const int q = fast_div(b, ln.mI), i = b - q * ln.I;
+  const int o = fast_div(q, mnb), j = q - o * nb;
+  const int jq = fast_div(j, mns), jm = j - jq * Ns;
+  return Butterfly{i, o, j, jq, jm};
+}
+
 // 6-point DFT as 2 x 3 (coprime: no twiddles), in place
 template <typename T> __device__ __forceinline__ void dft6(CX<T> *v, T s) {
   CX<T> e[3] = {v[0], v[2], v[4]}, o[3] = {v[3], v[5], v[1]};
@@ -178,16 +190,14 @@ __device__ __forceinline__ void pp_pass(const CX<T> *src, CX<T> *dst, int nb, co
                                         uint32_t mnb, uint32_t mns, const CX<T> *tw, T s) {
   const int total = ln.lines * nb, stride = nb / Ns;
   for (int b = threadIdx.x; b < total; b += blockDim.x) {
-    const int q = fast_div(b, ln.mI), i = b - q * ln.I;
-    const int o = fast_div(q, mnb), j = q - o * nb;
-    const int jq = fast_div(j, mns), jm = j - jq * Ns;
-    const CX<T> *x = src + i + o * ln.so;
+    const Butterfly at = butterfly(b, nb, ln, Ns, mnb, mns);
+    const CX<T> *x = src + at.i + at.o * ln.so;
     CX<T> v[R];
 #pragma unroll
     for (int k = 0; k < R; k++) {
-      CX<T> a = x[(j + k * nb) * ln.se];
-      if (k > 0 && jm > 0) {
-        CX<T> w = tw[jm * k * stride];
+      CX<T> a = x[(at.j + k * nb) * ln.se];
+      if (k > 0 && at.jm > 0) {
+        CX<T> w = tw[at.jm * k * stride];
         w.y *= s;
         a = cmul(a, w);
       }
@@ -195,7 +205,7 @@ __device__ __forceinline__ void pp_pass(const CX<T> *src, CX<T> *dst, int nb, co
     }
     if constexpr (R == 6) dft6<T>(v, s);
     else small_dft<R, T>(v, s);
-    CX<T> *y = dst + i + o * ln.so + (jq * Ns * R + jm) * ln.se;
+    CX<T> *y = dst + at.i + at.o * ln.so + (at.jq * Ns * R + at.jm) * ln.se;
 #pragma unroll
     for (int k = 0; k < R; k++) y[k * Ns * ln.se] = v[k];
   }
@@ -203,7 +213,13 @@ __device__ __forceinline__ void pp_pass(const CX<T> *src, CX<T> *dst, int nb, co
 }
 
 // a value every lane holds alike, in a scalar register
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__host__ __device__ __forceinline__ int uni(int v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_readfirstlane(v);
+#else
+  return v;
+#endif
+}
 
 // all passes of one transform of the lines at buf + r (r = 0 or FftCap, the
 // two buffers); returns the place of the result.  The passes, axes and directions are run
@@ -694,6 +710,90 @@ __device__ __forceinline__ void slab_spread(const BatchSys &S, const Ws<T> &w, c
   }
 }
 
+// The steps of grid_potential, as numbers: nf forward steps, nz of columns along
+// z, nf inverse.  A step holds in LDS either contiguous points [first, first + ne)
+// (slabs of np planes, rows), or L lines from `first` of an axis, element e of
+// line l at l + L e (columns; ne counts the places, lines past the end included).
+enum { SLAB, ROWS, YCOL, ZCOL };
+struct GridSteps {
+  int K0, K1, K2, P, Lx, Ly, Lz, pl, nx, ny, nz, nf;
+  bool slab;
+};
+__host__ __device__ __forceinline__ GridSteps grid_steps(const BatchSys &S) {
+  GridSteps G;
+  G.K0 = uni(S.K0);
+  G.K1 = uni(S.K1);
+  G.K2 = uni(S.K2);
+  G.P = uni(S.P);
+  const int nP = uni(S.nP);
+  G.Lx = uni(S.Lx);
+  G.Ly = uni(S.Ly);
+  G.Lz = uni(S.Lz);
+  G.pl = G.K0 * G.K1;
+  G.slab = G.P > 0;
+  G.nx = G.slab ? 0 : (G.K1 * G.K2 + G.Lx - 1) / G.Lx;
+  G.ny = G.slab ? 0 : (G.K0 * G.K2 + G.Ly - 1) / G.Ly;
+  G.nz = (G.pl + G.Lz - 1) / G.Lz;
+  G.nf = G.slab ? nP : G.nx + G.ny;
+  return G;
+}
+struct GridStep {
+  int view, c, inv, L, nl, first, ne, np;
+  uint32_t mL, mK0;
+};
+__host__ __device__ __forceinline__ GridStep grid_step(const GridSteps &G, int step, const uint32_t &mLy,
+                                                       const uint32_t &mLz, const uint32_t &mN0) {
+  int view, c, inv = 0;
+  if (step < G.nf) {
+    view = G.slab ? SLAB : (step < G.nx ? ROWS : YCOL);
+    c = view == YCOL ? step - G.nx : step;
+  } else if (step < G.nf + G.nz) {
+    view = ZCOL;
+    c = step - G.nf;
+  } else {
+    inv = 1;
+    c = step - G.nf - G.nz;
+    view = G.slab ? SLAB : (c < G.ny ? YCOL : ROWS);
+    if (view == ROWS) c -= G.ny;
+  }
+  const int L = view == YCOL ? G.Ly : G.Lz, N = view == YCOL ? G.K1 : G.K2, nl = view == YCOL ? G.K0 * G.K2 : G.pl;
+  const uint32_t mL = view == YCOL ? uni(mLy) : uni(mLz), mK0 = uni(mN0);
+  int first, ne, np = 0;
+  if (view == SLAB) {
+    np = G.P < G.K2 - c * G.P ? G.P : G.K2 - c * G.P;
+    first = c * G.P * G.pl;
+    ne = np * G.pl;
+  } else if (view == ROWS) {
+    const int left = G.K1 * G.K2 - c * G.Lx;
+    first = c * G.Lx * G.K0;
+    ne = (G.Lx < left ? G.Lx : left) * G.K0;
+  } else {
+    first = c * L;
+    ne = L * N;
+  }
+  return GridStep{view, c, inv, L, nl, first, ne, np, mL, mK0};
+}
+
+// grid point of place t of a step; ok: it has one
+__host__ __device__ __forceinline__ int step_place(const GridSteps &G, const GridStep &s, int t, bool &ok) {
+  ok = t < s.ne;
+  if (!(s.view >= YCOL)) return s.first + t;
+  const int e = fast_div(t, s.mL), q = s.first + t - e * s.L;
+  ok = ok && q < s.nl;
+  if (s.view == ZCOL) return q + G.pl * e;
+  const int z = fast_div(q, s.mK0);
+  return q - z * G.K0 + G.K0 * (e + G.K1 * z);
+}
+
+// the lines of axis ax that a step transforms
+__host__ __device__ __forceinline__ Lines step_lines(const GridSteps &G, const GridStep &s, int ax) {
+  Lines ln;
+  if (s.view >= YCOL) ln = Lines{s.L, 0, s.L, s.L, s.mL};
+  else if (ax == 0) ln = Lines{1, G.K0, 1, s.view == SLAB ? s.np * G.K1 : (int)fast_div(s.ne, s.mK0), 0u};
+  else ln = Lines{G.K0, G.pl, G.K0, s.np * G.K0, s.mK0};
+  return ln;
+}
+
 // Spread the sources into the system's grid and convolve it with the influence
 // function (un-normalised inverse, Complex.java:436-470); reads of the grid
 // may follow at once.  One step at a time goes through the two LDS buffers:
@@ -710,59 +810,19 @@ __device__ __forceinline__ void slab_spread(const BatchSys &S, const Ws<T> &w, c
 template <typename T, int NT, bool IND>
 __device__ void grid_potential(const BatchSys &S, const Ws<T> &w, const double *s0, const double *s1, CX<T> *buf,
                                const CX<T> *tw) {
-  const int K0 = uni(S.K0), K1 = uni(S.K1), K2 = uni(S.K2), P = uni(S.P), nP = uni(S.nP);
-  const int Lx = uni(S.Lx), Ly = uni(S.Ly), Lz = uni(S.Lz), pl = K0 * K1;
+  const GridSteps G = grid_steps(S);
+  const int K0 = G.K0, K1 = G.K1, K2 = G.K2, P = G.P, nf = G.nf, nz = G.nz;
   const T *recip = (const T *)(const void *)S.recip;
-  const bool slab = P > 0;
-  const int nx = slab ? 0 : (K1 * K2 + Lx - 1) / Lx, ny = slab ? 0 : (K0 * K2 + Ly - 1) / Ly;
-  const int nz = (pl + Lz - 1) / Lz, nf = slab ? nP : nx + ny;
-  if (!slab) {
+  if (!G.slab) {
     grid_zero<T, NT>(S, w);
     atomic_sync();
     grid_spread<T, NT, IND>(S, w, s0, s1);
     atomic_sync();
   }
-  enum { SLAB, ROWS, YCOL, ZCOL };
   for (int step = 0; step < 2 * nf + nz; step++) {
-    int view, c, inv = 0;
-    if (step < nf) {
-      view = slab ? SLAB : (step < nx ? ROWS : YCOL);
-      c = view == YCOL ? step - nx : step;
-    } else if (step < nf + nz) {
-      view = ZCOL;
-      c = step - nf;
-    } else {
-      inv = 1;
-      c = step - nf - nz;
-      view = slab ? SLAB : (c < ny ? YCOL : ROWS);
-      if (view == ROWS) c -= ny;
-    }
-    // contiguous steps: points [first, first + ne); columns: lines [first,
-    // first + cnt) of the axis, element e of line l in LDS at l + L e
-    const bool col = view >= YCOL;
-    const int L = view == YCOL ? Ly : Lz, N = view == YCOL ? K1 : K2, nl = view == YCOL ? K0 * K2 : pl;
-    const uint32_t mL = view == YCOL ? uni(S.mLy) : uni(S.mLz), mK0 = uni(S.rad[0].mN);
-    int first, ne, np = 0;
-    if (view == SLAB) {
-      np = min(P, K2 - c * P);
-      first = c * P * pl;
-      ne = np * pl;
-    } else if (view == ROWS) {
-      first = c * Lx * K0;
-      ne = min(Lx, K1 * K2 - c * Lx) * K0;
-    } else {
-      first = c * L;
-      ne = L * N;
-    }
-    auto place = [&](int t, bool &ok) -> int {
-      ok = t < ne;
-      if (!col) return first + t;
-      const int e = fast_div(t, mL), q = first + t - e * L;
-      ok = ok && q < nl;
-      if (view == ZCOL) return q + pl * e;
-      const int z = fast_div(q, mK0);
-      return q - z * K0 + K0 * (e + K1 * z);
-    };
+    const GridStep st = grid_step(G, step, S.mLy, S.mLz, S.rad[0].mN);
+    const int view = st.view, c = st.c, inv = st.inv, ne = st.ne, np = st.np;
+    auto place = [&](int t, bool &ok) -> int { return step_place(G, st, t, ok); };
     constexpr int MAXE = (FftCap<T>::value + NT - 1) / NT;
     CX<T> v[MAXE];
     if (view == SLAB && !inv) {
@@ -807,10 +867,7 @@ __device__ void grid_potential(const BatchSys &S, const Ws<T> &w, const double *
     for (int f = 0; f < nfft; f++) {
       const int ax = view == SLAB ? (f ^ inv) : (view == ROWS ? 0 : (view == YCOL ? 1 : 2));
       const T s = view == ZCOL ? (f ? (T)-1 : (T)1) : (inv ? (T)-1 : (T)1);
-      Lines ln;
-      if (col) ln = Lines{L, 0, L, L, mL};
-      else if (ax == 0) ln = Lines{1, K0, 1, view == SLAB ? np * K1 : (int)fast_div(ne, mK0), 0u};
-      else ln = Lines{K0, pl, K0, np * K0, mK0};
+      const Lines ln = step_lines(G, st, ax);
       if (f && view == ZCOL) {
         for (int t = threadIdx.x; t < ne; t += NT) {
           bool ok;
@@ -1252,6 +1309,8 @@ __device__ void run_system(const BatchSys &S, const BatchPrm &P, const Ws<T> &w,
 template <typename T, int NT, int LPA>
 __global__ void __launch_bounds__(NT) k_batch(const BatchSys *__restrict__ sys, int nsys, BatchPrm P,
                                                double *__restrict__ out, int *__restrict__ next) {
+  static_assert((2 * FftCap<T>::value + TW_CAP) * sizeof(CX<T>) + 16 * (NT / 64) * sizeof(double) + sizeof(BatchSys) +
+                        sizeof(Ws<T>) + sizeof(BatchPrm) + 16 <= 65536, "the workgroup's LDS exceeds 64 KB");
   __shared__ __align__(16) CX<T> buf[2 * FftCap<T>::value];
   __shared__ __align__(16) CX<T> tw[TW_CAP];
   __shared__ double red[16 * (NT / 64)];
@@ -1495,6 +1554,92 @@ static void pool_buffers(Pool *pl, std::vector<NbHandle *> &hs, const std::vecto
   b.tune = pl;
 }
 
+// slabs, lines per chunk and passes of the grid S.K0 x S.K1 x S.K2
+template <typename T>
+static void plan_grid(BatchSys &S) {
+  const int cap = FftCap<T>::value;
+  // chunks of nearly equal size, as few as the buffer allows
+  auto even = [](int total, int most) {
+    most = std::max(1, std::min(most, total));
+    const int chunks = (total + most - 1) / most;
+    return (total + chunks - 1) / chunks;
+  };
+  if (cap >= S.K0 * S.K1) {
+    S.P = even(S.K2, cap / (S.K0 * S.K1));
+    S.nP = (S.K2 + S.P - 1) / S.P;
+  }
+  S.Lx = even(S.K1 * S.K2, cap / S.K0);
+  S.Ly = even(S.K0 * S.K2, cap / S.K1);
+  S.Lz = even(S.K0 * S.K1, cap / S.K2);
+  S.mLy = div_magic(S.Ly);
+  S.mLz = div_magic(S.Lz);
+  const int K[3] = {S.K0, S.K1, S.K2};
+  for (int d = 0; d < 3; d++) S.rad[d] = batch_factor(K[d]);
+}
+
+// The steps of grid_potential on one grid, walked on the host with the kernel's
+// own schedule and index functions: what is wrong with them, or nothing.  slip:
+// a mistake to find (1 a plane too many in a slab, 2 a wrong magic number).
+template <typename T>
+static std::string walk_grid(int K0, int K1, int K2, int slip) {
+  BatchSys S;
+  memset(&S, 0, sizeof(S));
+  S.K0 = K0;
+  S.K1 = K1;
+  S.K2 = K2;
+  plan_grid<T>(S);
+  if (slip == 1) S.P++;
+  if (slip == 2) S.rad[0].mnb[0] /= 2;
+  const GridSteps G = grid_steps(S);
+  const int ntot = K0 * K1 * K2, cap = FftCap<T>::value;
+  std::vector<int> seen[2][4];
+  for (auto &d : seen)
+    for (auto &v : d) v.assign(ntot, 0);
+  for (int step = 0; step < 2 * G.nf + G.nz; step++) {
+    const GridStep st = grid_step(G, step, S.mLy, S.mLz, S.rad[0].mN);
+    if (st.ne <= 0 || st.ne > cap) return "a step exceeds the buffer";
+    if (st.view == SLAB && !st.inv && st.ne * sizeof(CX<double>) > 2 * cap * sizeof(CX<T>)) return "the slab's sums exceed the buffers";
+    for (int t = 0; t < st.ne; t++) {
+      bool ok;
+      const int g = step_place(G, st, t, ok);
+      if (!ok) continue;
+      if (g < 0 || g >= ntot) return "a point outside the grid";
+      seen[st.inv][st.view][g]++;
+    }
+    for (int ax = 0; ax < 3; ax++) {
+      if (st.view == SLAB ? ax == 2 : ax != st.view - 1) continue;
+      const Lines ln = step_lines(G, st, ax);
+      const Radices &rad = S.rad[ax];
+      const int N = ax == 0 ? K0 : (ax == 1 ? K1 : K2), tw0 = ax == 0 ? 0 : (ax == 1 ? K0 : K0 + K1);
+      int Ns = 1;
+      for (int p = 0; p < rad.nr; p++) {
+        const int R = rad.r[p], nb = N / R;
+        std::vector<int> rd(st.ne, 0), wr(st.ne, 0);
+        for (int b = 0; b < ln.lines * nb; b++) {
+          const Butterfly at = butterfly(b, nb, ln, Ns, rad.mnb[p], rad.mns[p]);
+          for (int k = 0; k < R; k++) {
+            const int base = at.i + at.o * ln.so, x = base + (at.j + k * nb) * ln.se,
+                      y = base + (at.jq * Ns * R + at.jm + k * Ns) * ln.se, w = at.jm * k * (nb / Ns);
+            if (x < 0 || x >= st.ne || y < 0 || y >= st.ne) return "an element outside the step's";
+            if (w < 0 || w >= N || tw0 + w >= TW_CAP) return "a twiddle outside its table";
+            rd[x]++;
+            wr[y]++;
+          }
+        }
+        for (int t = 0; t < st.ne; t++)
+          if (rd[t] != 1 || wr[t] != 1) return "an element not read and written once in a pass";
+        Ns *= R;
+      }
+      if (Ns != N) return "the passes do not make up the line";
+    }
+  }
+  for (int inv = 0; inv < 2; inv++)
+    for (int view = 0; view < 4; view++)
+      for (int n : seen[inv][view])
+        if (n != (view == ZCOL ? !inv : (G.slab == (view == SLAB)))) return "a point not taken once";
+  return "";
+}
+
 // One launch of the batch kernel over the systems in queue order, with the
 // buffers of b (workspace offsets off).  Returns 1 when some rows overflowed
 // (their capacities are raised; the batch must be repeated).
@@ -1513,25 +1658,7 @@ static int run_batch(BatchBuf &bf, std::vector<NbHandle *> &hs, BatchPrm &P, std
     S.K2 = h->prm.do_pme ? h->K[2] : 1;
     S.maxa = h->fmaxa;
     S.maxb = h->fmaxb;
-    if (h->prm.do_pme) {
-      const int cap = FftCap<T>::value;
-      // chunks of nearly equal size, as few as the buffer allows
-      auto even = [](int total, int most) {
-        most = std::max(1, std::min(most, total));
-        const int chunks = (total + most - 1) / most;
-        return (total + chunks - 1) / chunks;
-      };
-      if (cap >= S.K0 * S.K1) {
-        S.P = even(S.K2, cap / (S.K0 * S.K1));
-        S.nP = (S.K2 + S.P - 1) / S.P;
-      }
-      S.Lx = even(S.K1 * S.K2, cap / S.K0);
-      S.Ly = even(S.K0 * S.K2, cap / S.K1);
-      S.Lz = even(S.K0 * S.K1, cap / S.K2);
-      S.mLy = div_magic(S.Ly);
-      S.mLz = div_magic(S.Lz);
-      for (int d = 0; d < 3; d++) S.rad[d] = batch_factor(h->K[d]);
-    }
+    if (h->prm.do_pme) plan_grid<T>(S);
     S.lcut = std::max(h->prm.ewald_cutoff, h->prm.vdw_cutoff) + h->prm.list_buffer;
     S.cell = h->cell;
     S.cell.multi = 1;
@@ -1891,6 +2018,19 @@ int nb_batch_last_config(int device, int32_t cfg[4], double *kernel_ms) {
   for (int q = 0; q < 4; q++) cfg[q] = pl->last[q];
   if (kernel_ms) *kernel_ms = pl->last_ms;
   return NB_OK;
+}
+
+// walk_grid of one grid in one form (test entry): 0, or 1 with what is wrong
+extern "C" int nb_test_batch_walk(int K0, int K1, int K2, int precision, int slip, char *why, int cap) {
+  std::string s = "an edge that no grid has";
+  try {
+    if (std::min(K0, std::min(K1, K2)) >= 8 && std::max(K0, std::max(K1, K2)) <= 64)
+      s = precision == NB_PREC_MIXED ? walk_grid<float>(K0, K1, K2, slip) : walk_grid<double>(K0, K1, K2, slip);
+  } catch (std::exception &e) {
+    s = e.what();
+  }
+  if (why && cap > 0) snprintf(why, cap, "%s", s.c_str());
+  return s.empty() ? 0 : 1;
 }
 
 // nb_evaluate_batch with the batch kernel's shape given (test entry): -1 past

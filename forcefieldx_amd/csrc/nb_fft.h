@@ -21,7 +21,13 @@ __device__ __forceinline__ int wrapg(int i, int n) { return i >= n ? i - n : (i 
 __host__ __device__ __forceinline__ uint32_t div_magic(int d) {
   return d > 1 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u;
 }
-__device__ __forceinline__ int fast_div(int n, uint32_t m) { return m ? (int)__umulhi((uint32_t)n, m) : n; }
+__host__ __device__ __forceinline__ int fast_div(int n, uint32_t m) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return m ? (int)__umulhi((uint32_t)n, m) : n;
+#else
+  return m ? (int)(((uint64_t)(uint32_t)n * m) >> 32) : n;
+#endif
+}
 
 // radix of each pass over a line of N, with the magic numbers of its butterfly
 // count N / R and of the transforms' length Ns before it

@@ -1,86 +1,66 @@
 """LDS index bounds of the batch kernel's grid transforms, checked on the CPU.
 
-The batch kernel transforms each cell's grid through two LDS buffers of
-FftCap complex entries (28672 B each: 3584 FP32 or 1792 FP64 entries) and a
-twiddle table of TW_CAP = 3 x 64 entries.  A chunk of L lines of length N
-(L = max(1, min(FftCap / N, lines of the axis))) is loaded, passed through the
-out-of-place Stockham passes of N's radix schedule (4, 2, 3, 5, 7 in that
-order) and stored.  For every grid edge the batch path admits (at most 64,
-factors 2, 3, 5, 7) and every number of lines an axis can have (the product
-of two admitted edges), this walks every chunk and every butterfly of every
-pass and asserts that each LDS read, write and twiddle index is inside its
-buffer: the index arithmetic itself cannot run past the buffers, for any
-cell shape and for any of the tuner's workgroup sizes (they change only the
-thread stride of the same index set).
-"""
-import itertools
+The batch kernel transforms each cell's grid through two LDS buffers (28672 B
+each: 3584 FP32 or 1792 FP64 complex entries) and a twiddle table of 3 x 64
+entries.  The library walks a grid on the host with the schedule it hands to
+the kernel and the index functions the kernel is compiled from
+(nb_test_batch_walk): every step (slabs of whole planes, rows and columns of
+planes that exceed a buffer, columns along z) and every butterfly of every
+pass.  Each LDS read, write and twiddle index stays inside its buffer, each
+element is read and written once in a pass, each grid point is taken once in
+each direction.  The tuner's workgroup sizes change only the thread stride of
+the same index set.  The sum of a workgroup's static LDS (63,288 B at most) is
+asserted where the kernel is compiled."""
+import ctypes
 
 import numpy as np
+import pytest
+
+from forcefieldx_amd import ffi
 
 
 def radices(n):
-    """The radix schedule of nb_factor: fours, then twos, threes, fives, sevens;
-    None when n has another prime factor."""
+    """The prime factors of n among 2, 3, 5 and 7; None when it has another."""
     r = []
-    for p in (4, 2, 3, 5, 7):
+    for p in (2, 3, 5, 7):
         while n % p == 0:
             r.append(p)
             n //= p
     return r if n == 1 else None
 
 
-ADMITTED = [k for k in range(2, 65) if radices(k) is not None]
-FFT_CAP = {"float": 28672 // 8, "double": 28672 // 16}
+# the edges the batch path admits (at least 8 for any grid, at most 64 for this kernel)
+ADMITTED = [k for k in range(8, 65) if radices(k) is not None]
 TW_CAP = 3 * 64
 
 
-def pass_indices(N, nlines, line_fast, R, Ns):
-    """Every (read, write, twiddle) index of one pp_pass, vectorised over the
-    butterflies b < nlines * N / R (sl = N, se = 1 for rows; sl = 1, se =
-    nlines for interleaved lines)."""
-    nb = N // R
-    stride = N // (Ns * R)
-    sl, se = (1, nlines) if line_fast else (N, 1)
-    b = np.arange(nlines * nb)
-    if line_fast:
-        line, j = b % nlines, b // nlines
-    else:
-        j, line = b % nb, b // nb
-    jm = j % Ns
-    k = np.arange(R)[:, None]
-    reads = line * sl + (j + k * nb) * se
-    writes = line * sl + ((j // Ns) * Ns * R + jm + k * Ns) * se
-    tw = jm * k * stride
-    return reads, writes, tw
+def walk(grid, precision, slip=0):
+    why = ctypes.create_string_buffer(200)
+    rc = ffi.load().nb_test_batch_walk(*map(int, grid), precision, slip, why, len(why))
+    return rc, why.value.decode()
 
 
-def test_radix_schedules_match_the_admitted_edges():
+def test_admitted_edges():
     assert 64 in ADMITTED and 49 in ADMITTED and 11 not in ADMITTED and 22 not in ADMITTED
-    for n in ADMITTED:
-        assert int(np.prod(radices(n))) == n
 
 
-def test_every_lds_index_of_the_batch_transforms_is_in_bounds():
-    products = sorted({a * b for a, b in itertools.combinations_with_replacement(ADMITTED, 2)})
-    for real, cap in FFT_CAP.items():
-        for N in ADMITTED:
-            for P in products:
-                L = max(1, min(cap // N, P))
-                # a chunk of cnt <= L lines: load / store indices t < cnt * N
-                assert L * N <= cap, (real, N, P)
-                for cnt in {L, P % L} - {0}:
-                    for line_fast in (False, True):
-                        Ns = 1
-                        for R in radices(N):
-                            rd, wr, tw = pass_indices(N, cnt, line_fast, R, Ns)
-                            assert rd.min() >= 0 and rd.max() < cnt * N <= cap, (real, N, P, cnt, R, Ns)
-                            assert wr.min() >= 0 and wr.max() < cnt * N <= cap, (real, N, P, cnt, R, Ns)
-                            # every element of the chunk is written exactly once per pass
-                            assert np.unique(wr).size == cnt * N, (real, N, P, cnt, R, Ns)
-                            assert tw.max() < N <= 64, (N, R, Ns)
-                            Ns *= R
+@pytest.mark.parametrize("precision", [ffi.NB_PREC_FP64, ffi.NB_PREC_MIXED], ids=["fp64", "mixed"])
+def test_every_lds_index_of_the_batch_transforms_is_in_bounds(precision):
+    # every plane, with the z edges taken in turn, and every z edge on the smallest and largest planes
+    grids = [(a, b, ADMITTED[(7 * i + j) % len(ADMITTED)]) for i, a in enumerate(ADMITTED) for j, b in enumerate(ADMITTED)]
+    grids += [(a, b, c) for c in ADMITTED for a, b in ((8, 8), (8, 64), (64, 8), (64, 64), (42, 42), (42, 45))]
+    for grid in grids:
+        assert walk(grid, precision) == (0, ""), grid
+
+
+@pytest.mark.parametrize("precision", [ffi.NB_PREC_FP64, ffi.NB_PREC_MIXED], ids=["fp64", "mixed"])
+def test_the_walk_finds_mistakes(precision):
+    """A plane too many in a slab, a wrong magic number, edges no grid has."""
+    for grid in ((32, 28, 63), (24, 18, 48)):
+        assert walk(grid, precision, 1)[0] == walk(grid, precision, 2)[0] == 1, grid
+    assert walk((22, 16, 16), precision)[0] == walk((7, 16, 16), precision)[0] == walk((16, 70, 16), precision)[0] == 1
 
 
 def test_twiddle_tables_of_three_axes_fit():
     # the three axes' tables are stored one after the other: K0 + K1 + K2 <= 3 x 64
-    assert 3 * max(ADMITTED) <= TW_CAP
+    assert 3 * max(ADMITTED) <= TW_CAP and np.prod(radices(max(ADMITTED))) == 64

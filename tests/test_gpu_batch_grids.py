@@ -111,9 +111,10 @@ def test_shape_past_the_last():
 
 
 def test_slab_transforms_stay_in_the_buffer():
-    """The LDS indexes of a slab's x and y passes, for every plane of admitted
-    edges that fits: each pass reads and writes every point exactly once, and
-    the magic numbers divide exactly."""
+    """A model of a slab's x and y passes, independent of the library's code
+    (which test_batch_lds_bounds.py walks): for every plane of admitted edges that
+    fits, each pass reads and writes every point exactly once, and magic numbers
+    as the library makes them divide exactly."""
     def radices(n):
         r = []
         for p in (4, 2, 3, 5, 7):
