@@ -594,9 +594,12 @@ void nb_perm_field(NbHandle *h) {
 // launch at 20,736 atoms, 250 -> 159 us at 90,003.  The slots, 16 bytes a row
 // entry, grow with the rows' capacity, outside a recording (a recorded
 // evaluation has the capacities of the regular one before it).  They are an
-// option: a size that does not fit a quarter of the free memory, so that rows
-// and other handles find theirs (a cluster without a cutoff has n^2 entries), is
-// not asked for again, and the factors are formed each time.
+// option: a size that cannot be had is not asked for again, and the factors are
+// formed each time.  From 64 MB on they may take a quarter of the free memory, so
+// that rows and other handles find theirs (a cluster without a cutoff has n^2
+// entries); below, the question alone would cost a tenth of a small handle's
+// first evaluation (648 atoms 1.37 -> 1.55 ms).
+constexpr size_t NB_COEF_ASK = (size_t)64 << 20;
 int nb_coef_mode(NbHandle *h) {
   if (h->prm.precision == NB_PREC_MIXED) return NB_DIP_FORM;
   const size_t bytes = sizeof(DipCoef<double>) * (size_t)h->n * h->maxew;
@@ -606,7 +609,8 @@ int nb_coef_mode(NbHandle *h) {
     h->d_ewcoef = nullptr;
     h->ewcoef_cap = 0;
     size_t avail = 0, total = 0;
-    if (hipMemGetInfo(&avail, &total) != hipSuccess || bytes > avail / 4 || hipMalloc(&h->d_ewcoef, bytes) != hipSuccess) {
+    const bool room = bytes < NB_COEF_ASK || (hipMemGetInfo(&avail, &total) == hipSuccess && bytes <= avail / 4);
+    if (!room || hipMalloc(&h->d_ewcoef, bytes) != hipSuccess) {
       h->d_ewcoef = nullptr;
       h->ewcoef_refused = bytes;
       (void)hipGetLastError();

@@ -30,8 +30,8 @@ def stub(library, monkeypatch):
     assert s.faults() == [] and s.counts()["live"] == s.kept
 
 
-def handle(precision, grid=PARAMS.grid):
-    xyz, box, top = water_box(216, 18.643, seed=1)
+def handle(precision, grid=PARAMS.grid, waters=216):
+    xyz, box, top = water_box(waters, 18.643 * (waters / 216) ** (1.0 / 3.0), seed=1)
     h = ffi.Handle(ffi.params_from(PARAMS, grid, precision), top)
     h.set_cell(box)
     h.set_positions(xyz)
@@ -99,21 +99,24 @@ def test_lds_of_the_longest_lines(stub, precision, edge):
 def test_radial_factors_are_an_option(stub):
     """The FP64 form's stored radial factors (16 bytes a row entry, its largest
     allocation here) are tried once per row capacity and left out when they
-    fail or would take more than a quarter of the free memory."""
-    h, _, _ = handle(ffi.NB_PREC_FP64)
-    h.evaluate(ffi.NB_GRAD)   # the rows' capacities
-    h.close()
-    size = max(stub.allocations())
-    assert size % (16 * h.n) == 0
-    for kw, tries in ((dict(fail_bytes=size), 1), (dict(free_bytes=4 * size - 1), 0)):
-        h, _, _ = handle(ffi.NB_PREC_FP64)
-        stub.set(**kw)
+    fail or, from 64 MB on, would take more than a quarter of the free memory."""
+    for waters in (216, 6912):
+        h, _, _ = handle(ffi.NB_PREC_FP64, waters=waters)
         stub.reset()
-        for _ in range(3):
-            h.evaluate(ffi.NB_GRAD)
-        assert stub.counts()["failed"] == tries and max(stub.allocations()) < size
+        h.evaluate(ffi.NB_GRAD)   # the rows' capacities
         h.close()
-        stub.set()
+        size = max(stub.allocations())
+        assert size % (16 * h.n) == 0 and (size >= 64 << 20) == (waters == 6912)
+        for kw, tries, held in ((dict(fail_bytes=size), 1, False),
+                                (dict(free_bytes=4 * size - 1), 0, waters == 216)):
+            h, _, _ = handle(ffi.NB_PREC_FP64, waters=waters)
+            stub.set(**kw)
+            stub.reset()
+            for _ in range(3):
+                h.evaluate(ffi.NB_GRAD)
+            assert stub.counts()["failed"] == tries and (size in stub.allocations()) == held
+            h.close()
+            stub.set()
 
 
 @FORMS
