@@ -15,15 +15,30 @@ pytestmark = pytest.mark.gpu
 DENSITY = 6912 / 59.1 ** 3
 
 
-@pytest.mark.parametrize("waters, edge, grid", [(400, 1.0, 16), (1500, 1.0, 12), (1500, 2.1, 16)])
-def test_crowded_bricks(oracle, waters, edge, grid):
+def brick_counts(xyz, box, grid):
+    """Atoms per brick of a cubic cell: an atom belongs to the brick of its first
+    spline point, four before the point of its coordinate (measured from the cell's
+    centre); an axis of 16 points or fewer has two bricks."""
+    w = xyz.reshape(-1, 3) / box[0]
+    u = w - np.floor(w + 0.5) + 0.5
+    start = ((grid * u).astype(int) - 4) % grid
+    brick = ((start + 1) * 2 - 1) // grid
+    return np.bincount(brick @ [1, 2, 4], minlength=8)
+
+
+# more atoms in a brick than a pass stages; then, in a cell of 2.3 times the water's edge with the
+# water in its middle, all in one brick and more than the sums hold at the finest quantum
+@pytest.mark.parametrize("waters, edge, grid, most", [(400, 1.0, 16, 128), (1500, 1.0, 12, 128), (1500, 2.3, 16, 4096)])
+def test_crowded_bricks(oracle, waters, edge, grid, most):
     """FP64 reciprocal energy and gradient on coarse grids against the oracle
-    (1e-8), the mixed form within its 1e-5 of them; in a cell of twice the
-    water's edge all atoms lie in one of the eight bricks."""
+    (1e-8), the mixed form within its 1e-5 of them."""
     length = (waters / DENSITY) ** (1.0 / 3.0)
     xyz, box, top = water_box(waters, length, seed=7)
     box = np.array(box, float)
     box[:3] *= edge
+    xyz = xyz + 0.5 * (edge - 1.0) * length
+    counts = brick_counts(xyz, box, grid)
+    assert counts.sum() == top.n and counts.max() > most
     p = NonbondedParams(ewald_cutoff=5.0, vdw_cutoff=5.0, polarization=0, grid=(grid, grid, grid))
     eo, go, _, _ = oracle.evaluate(oracle.System(xyz, box, top), p)
     for precision, tol in ((ffi.NB_PREC_FP64, 1e-8), (ffi.NB_PREC_MIXED, 1e-5)):
