@@ -165,7 +165,7 @@ __device__ __forceinline__ void spread_source(const double *__restrict__ fmp, co
 // binned in its brick into an LDS brick of edge ext (its points plus the
 // 4-point spill into the next bricks) and stores it, in the grid's real type,
 // to the brick buffer; the forward x transform assembles each grid point from
-// its own brick and the spills of up to 7 previous bricks (brick_point), in a
+// its own brick and the spills of up to 7 previous bricks (brick_points), in a
 // fixed order.  Thread (atom, ky, kz) forms the y-z weight and adds 5
 // consecutive x points; what the 25 threads of an atom share (its place in the
 // brick and its source) is worked out once by the pass over the bin that finds
@@ -343,9 +343,10 @@ __global__ void __launch_bounds__(256) k_spread_brick(int n, Bricks bk, const in
 // the r.z partial sums.  As two launches on two streams they cost a fork and a
 // join of the queues per solver iteration, 5-10 us each, beside ~75 us of
 // kernels at 20,736 atoms.  Workgroups come in groups of 8, one per XCD; the
-// spread's groups lead while all workgroups are resident together (its chain
-// is the longer one), otherwise the two kinds alternate in proportion, so that
-// the LDS-bound and the gather-bound ones share the compute units.
+// spread's groups lead (its chain is the longer one) in a launch of at most four
+// workgroups a compute unit, which are resident together but for the FP64 kernels
+// that form the factors (three); otherwise the two kinds alternate in proportion,
+// so that the LDS-bound and the gather-bound ones share the compute units.
 struct FieldArgs {
   const uint32_t *lst;
   const int32_t *cnt;
@@ -1268,9 +1269,16 @@ static void spread_field_into(NbHandle *h, const double *u, const double *up, co
   FieldArgs F{h->d_ew, h->d_new, h->maxew, use_recip ? h->prm.ewald_alpha : 0.0, f, fp};
   TotalsArgs R{h->d_part, h->part_stride, nrz, h->d_scal};
   const int front = (gs + gf) * NB_XCD <= 4 * 256 ? 1 : 0;
-  NB_LAUNCH((k_spread_brick_k_dip_field<T, NB_LPA_PCG, MODE>), dim3((gs + gf + (nrz > 0 ? 1 : 0)) * NB_XCD), dim3(256),
-            0, h->n, bricks_of(h), h->nbricks, h->d_bstart, h->d_batom, theta, h->d_igrid, u, up, frac_of(h),
-            (T *)h->d_bbuf, gs, gf, front, (const DipRec<T> *)rec, F, h->cell, (DipCoef<T> *)h->d_ewcoef, R, h->ctl);
+  const dim3 G((gs + gf + (nrz > 0 ? 1 : 0)) * NB_XCD);
+  // the profiler's names tell the two arithmetics apart: a solve of the mixed
+  // form launches both
+#define NB_SF(KERNEL)                                                                                                  \
+  NB_LAUNCH(KERNEL, G, dim3(256), 0, h->n, bricks_of(h), h->nbricks, h->d_bstart, h->d_batom, theta, h->d_igrid, u, up, \
+            frac_of(h), (T *)h->d_bbuf, gs, gf, front, (const DipRec<T> *)rec, F, h->cell, (DipCoef<T> *)h->d_ewcoef, R, \
+            h->ctl)
+  if constexpr (sizeof(T) == sizeof(float)) NB_SF((k_spread_brick_k_dip_field<float, NB_LPA_PCG, MODE>));
+  else NB_SF((k_spread_brick_k_dip_field<double, NB_LPA_PCG, MODE>));
+#undef NB_SF
 }
 
 static bool mixed_grid(const NbHandle *h) { return h->prm.precision == NB_PREC_MIXED; }
