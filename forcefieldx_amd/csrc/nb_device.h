@@ -46,8 +46,9 @@ __device__ __forceinline__ void entry_shift(const CellD &c, uint32_t en, double 
 // minimum image with the reference's independent fractional rounding (image
 // sums: the displacement already holds its translation).  The lattice
 // translation is subtracted from the Cartesian displacement, so a pair that
-// needs none keeps it unrounded; at a half-integer offset, where the reference
-// rounds away from zero, either image is equally far.  9 FP64 instructions in a
+// needs none keeps it unrounded.  At a half-integer offset, where the reference
+// rounds away from zero, the other image may be taken: both are half a cell width
+// or more away, beyond the cutoffs (a thinner cell takes image sums).  9 FP64 instructions in a
 // right-angled cell and 15 otherwise, in every pair kernel (transforming to
 // fractional coordinates and back takes 27).
 __device__ __forceinline__ double image(const CellD &c, double &dx, double &dy, double &dz) {

@@ -299,9 +299,10 @@ __device__ __forceinline__ void gather_atom(int s, int lane, bool valid, const T
     // PREFETCH (FP32 grids; in FP64 the registers spill): the 25 grid values of
     // the lane's plane are loaded before the first is used, one memory latency
     // instead of five, and two points in one 16-byte load unless a stencil of the
-    // wave crosses the cell's edge, 15 loads instead of 25 for the address unit,
-    // which bounds the gather.  An evaluation at 288,000 atoms mixed 9.66 -> 9.52
-    // ms, 20,736 1.127 -> 1.119
+    // wave crosses the cell's edge, 15 loads instead of 25 for the address unit.
+    // Neither gains by itself (an evaluation at 288,000 atoms mixed: 9.66 ms with
+    // neither, 9.67 paired, 9.70 early), together they do: 9.51, and 1.160 -> 1.151
+    // at 20,736
     CX<T> pre[PREFETCH ? 5 : 1][PREFETCH ? 5 : 1];
     if constexpr (PREFETCH) {
       typedef T pair_t __attribute__((ext_vector_type(4), aligned(sizeof(CX<T>))));
