@@ -62,3 +62,9 @@ class Stub:
 
     def faults(self):
         return self.L.stub_faults().decode().splitlines()
+
+    def taken_faults(self):
+        """The faults so far, which are then forgotten."""
+        f = self.faults()
+        self.L.stub_forget()
+        return f

@@ -216,6 +216,7 @@ long stub_allocations(long *out, long most) {
   return (long)sizes.size();
 }
 const char *stub_faults() { return faults.c_str(); }
+void stub_forget() { faults.clear(); }
 
 void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
 void __hipUnregisterFatBinary(void **) {}

@@ -1,6 +1,8 @@
 """What the library's host code asks the HIP runtime for, on a runtime without
 a device (host_stub): graphs, streams, events and memory are used within the
 runtime's rules, and dynamics records no graph."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -36,6 +38,52 @@ def handle(precision, grid=PARAMS.grid, waters=216):
     h.set_cell(box)
     h.set_positions(xyz)
     return h, xyz, np.ones(top.n)
+
+
+def test_misuse_is_found(stub):
+    """The runtime's model by itself: what the other tests rely on it to report."""
+    L, v = stub.L, ctypes.c_void_p
+    for f in ("hipMemcpyAsync", "hipMemsetAsync", "hipStreamWaitEvent", "hipEventRecord", "hipStreamBeginCapture",
+              "hipStreamEndCapture", "hipGraphInstantiate", "hipGraphLaunch", "hipGraphExecDestroy", "hipGraphDestroy",
+              "hipStreamSynchronize", "hipStreamDestroy", "hipEventDestroy", "hipFree", "hipMalloc"):
+        getattr(L, f).argtypes = None
+    a, b, e, p, g, x = v(), v(), v(), v(), v(), v()
+    L.hipStreamCreate(ctypes.byref(a)), L.hipStreamCreate(ctypes.byref(b)), L.hipEventCreate(ctypes.byref(e))
+    L.hipMalloc(ctypes.byref(p), ctypes.c_size_t(64))
+
+    def work(stream, nbytes=32):
+        L.hipMemcpyAsync(p, v(p.value + 32), ctypes.c_size_t(nbytes), 3, stream)   # device to device
+
+    def record(joined=True, body=None):
+        L.hipStreamBeginCapture(a, 0)
+        work(a)
+        L.hipEventRecord(e, a), L.hipStreamWaitEvent(b, e, 0)
+        work(b)
+        if body:
+            body()
+        if joined:
+            L.hipEventRecord(e, b), L.hipStreamWaitEvent(a, e, 0)
+        L.hipStreamEndCapture(a, ctypes.byref(g))
+        return stub.taken_faults()
+
+    assert record() == []
+    L.hipGraphInstantiate(ctypes.byref(x), g, None, None, ctypes.c_size_t(0))
+    L.hipGraphLaunch(x, a)
+    L.hipGraphExecDestroy(x)
+    assert stub.taken_faults() == ["a graph destroyed while a launch of it is outstanding"]
+    L.hipStreamWaitEvent(b, e, 0)
+    assert stub.taken_faults() == ["a wait for an event of a capture that has ended"]
+    L.hipGraphDestroy(g)
+    for joined, body, found in ((False, None, "a captured stream is not joined"),
+                                (True, lambda: L.hipStreamSynchronize(a), "hipStreamSynchronize inside a capture"),
+                                (True, lambda: L.hipMemsetAsync(p, 0, ctypes.c_size_t(8), a), "hipMemsetAsync in a captured graph")):
+        assert found in record(joined, body), found
+        L.hipGraphDestroy(g)
+    work(a, 64)
+    assert stub.taken_faults() == ["copy past the end of a device allocation (read)"]
+    L.hipGraphDestroy(g)
+    assert stub.taken_faults() == ["a graph destroyed that does not exist"]
+    L.hipFree(p), L.hipEventDestroy(e), L.hipStreamDestroy(a), L.hipStreamDestroy(b)
 
 
 @FORMS
